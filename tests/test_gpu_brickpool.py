@@ -106,6 +106,38 @@ def test_list_and_slot_counts_around_a_mask(yx, oracle_mod, cuda, cap, k):
         same()
 
 
+@pytest.mark.parametrize("cap", [126976, 126977, 209715, 2097152, 2097217])
+def test_pools_of_many_slots(yx, oracle_mod, cuda, cap):
+    """Slot counts around those where the sum of the used slots (31 chunks of
+    4096 items) and the scans of the slots' and the list's masks (32,768 masks
+    of 64) need more space or another path; half of the slots used before."""
+    torch = cuda
+    grid = 64 if cap < 64 ** 3 else 136
+    nb = grid ** 3
+    dev = torch.device("cuda", 0)
+    rng = np.random.default_rng(cap)
+    order = rng.permutation(nb).astype(np.int32)
+    start = np.full(nb, -1, np.int32)
+    start[order[:cap // 2]] = rng.permutation(cap)[:cap // 2]
+    table = torch.from_numpy(start).to(dev)
+    params = torch.zeros((cap, 4), dtype=torch.float32, device=dev)
+    pool = yx.composite.BrickPool(table, params, grid, 1)
+    orc = oracle_mod.BrickPoolOracle(start, np.zeros((cap, 4), np.float32), 1)
+    assert pool.stats() == (cap // 2, cap)
+    gone = order[:cap // 4]
+    assert pool.release(torch.from_numpy(gone).to(dev)) == orc.release(gone) == cap // 4
+    fresh = order[cap // 8:cap // 8 + cap]  # some have a slot, the others take every free one
+    slots, new = pool.alloc(torch.from_numpy(fresh).to(dev))
+    exp_slots, exp_new = orc.alloc(fresh)
+    assert new == exp_new and np.array_equal(slots.cpu().numpy(), exp_slots)
+    assert np.array_equal(table.cpu().numpy(), orc.table)
+    assert pool.stats() == (int(orc.used.sum()), cap)
+    values = rng.standard_normal((fresh.size, 4)).astype(np.float32)
+    pool.update(torch.from_numpy(fresh).to(dev), torch.from_numpy(values).to(dev))
+    orc.params[exp_slots] = values  # every listed brick has a slot of its own
+    assert np.array_equal(params.cpu().numpy(), orc.params)
+
+
 def test_existing_table_and_bad_table(yx, cuda):
     torch = cuda
     vol = yx.composite.Volume(64, 8, occupancy=0.2, seed=3)

@@ -252,9 +252,10 @@ static int bp_alloc(T** p, size_t n) {
 
 static uint32_t bp_masks(uint32_t n) { return n / 64u + (n % 64u ? 1u : 0u); }
 
-// Scan space for masks of `n` items, or of the slots.
-static int bp_scan_space(yx_brick_pool* p, uint32_t n) {
-    const size_t bytes = scan_workspace_bytes(std::max(bp_masks(std::max(n, p->vol.num_slots)), 1u));
+// Space for a scan or a sum of `items` items: a pool's creation sums the used
+// slots themselves, the calls scan masks of 64 slots or list entries.
+static int bp_scan_space(yx_brick_pool* p, uint32_t items) {
+    const size_t bytes = scan_workspace_bytes(std::max(items, 1u));
     if (bytes <= p->scan_bytes) return YX_OK;
     if (p->scan_tmp) BP_HIP(hipFree(p->scan_tmp));
     p->scan_tmp = nullptr;
@@ -359,7 +360,7 @@ static int ensure_list(yx_brick_pool* p, uint32_t n) {
     p->cap_masks = 0;
     int rc;
     if ((rc = bp_alloc(&p->d_new_mask, masks)) != YX_OK || (rc = bp_alloc(&p->d_new_before, masks)) != YX_OK ||
-        (rc = bp_scan_space(p, n)) != YX_OK)
+        (rc = bp_scan_space(p, masks)) != YX_OK)
         return rc;
     p->cap_masks = masks;
     return YX_OK;
