@@ -127,6 +127,51 @@ def test_samples_of_far_and_axis_aligned_rays(yx, oracle_mod, cuda, grid, brick)
     assert np.array_equal(ns.cpu().numpy().view(np.uint32), o_ns)
 
 
+@pytest.mark.parametrize("grid,brick,opaque,w,h", [
+    (32, 8, 0.1, 48, 40),      # four waves to a cell
+    (128, 8, 0.1, 64, 48),     # more than 2048 cells: a wave to each
+    (16, 8, 0.4, 300, 260),    # cells of several chunks of segments
+    (64, 8, 0.1, 300, 260),    # cells of one chunk
+    (32, 16, 0.1, 48, 40),
+    (32, 2, 0.1, 48, 40),      # segments of at most 8 samples
+])
+def test_gradient_of_occluded_voxels(yx, oracle_mod, cuda, grid, brick, opaque, w, h):
+    """Opacity gradients of voxels that light reaches only through opaque ones
+    (raw = 20: 2e-9 of it passes), against the FP64 reference and on their own
+    scale. What is left of a ray's colour behind sample k is the final colour
+    minus the forward's own prefix. An addition to the prefix is off by no more
+    than what it adds (the prefix itself is as near), so what is left is off by
+    no more than itself: by T_{k+1}, colours being in [0, 1]. dL/draw is then off by alpha |g| T_{k+1} a ray at
+    most, below the sum of the voxel's own colour gradients, alpha T_k g each
+    (g > 0 here); 1e-3 of that covers the rounding of everything else. 1e-13:
+    the reference's own difference of doubles."""
+    torch = cuda
+    rng = np.random.default_rng(grid + brick)
+    slots = (grid // brick) ** 3
+    table = rng.permutation(slots).astype(np.int32)
+    params = rng.random((grid ** 3, 4)).astype(np.float32)
+    params[:, 0] = np.where(rng.random(grid ** 3) < opaque, 20.0, -1.0)
+    views = yx.composite.orbit_views(1, 60.0, w, h, seed=2)
+    dev = torch.device("cuda", 0)
+    table_d, params_d, views_d = (torch.from_numpy(x).to(dev) for x in (table, params, views))
+    comp = yx.composite.Compositor()
+    rgb, _, ns = comp.forward(table_d, params_d, grid, brick, views_d, w, h)
+    target = np.full((1, h, w, 3), -0.5, np.float32)
+    grad = comp.backward(table_d, params_d, grid, brick, views_d, w, h, rgb, ns, 2.0 * (rgb + 0.5))
+    torch.cuda.synchronize()
+    grad = grad.cpu().numpy().astype(np.float64)
+    scale = grad[:, 1:].sum(1)
+    dim = np.nonzero((scale > 1e-12) & (scale < 1e-7))[0]
+    assert dim.size >= 100
+    sel = rng.choice(dim, size=min(512, dim.size), replace=False)
+    _, ref, _ = oracle_mod.CompositeOracle().grad(table, params, grid, brick, views, w, h, target, sel, max_rays=1,
+                                                  threads=8)
+    np.testing.assert_allclose(grad[sel, 1:], ref[:, 1:], rtol=1e-3)
+    err = np.abs(grad[sel, 0] - ref[:, 0])
+    bound = 1.001 * ref[:, 1:].sum(1) + 1e-13
+    assert (err <= bound).all(), f"{int((err > bound).sum())} of {sel.size} off, up to {(err / bound).max():.1f} bounds"
+
+
 def test_composite_512_full(yx, oracle_mod, cuda):
     """The full workload: 512^3 as 8^3 bricks at ~10 % occupancy, 16 views of
     512x512 rays; forward checked on every ray, gradient on 256 voxels."""
