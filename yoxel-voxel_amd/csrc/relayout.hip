@@ -480,12 +480,11 @@ int gpu_relayout(const uint32_t* d_vox, uint32_t nn, uint32_t root, void* stream
     uint32_t* d_lod = *lod_io;
     // bottom-up subtree sums: two buffers of 5 u64 per node of the widest level
     if (w->cap_wide < widest) {
-        size_t c = w->cap_wide * 5;
-        if ((rc = rl_grow(&w->sa, &c, (size_t)widest * 5, "subtree sums")) != YX_OK) return rc;
-        c = w->cap_wide * 5;
-        if ((rc = rl_grow(&w->sb, &c, (size_t)widest * 5, "subtree sums")) != YX_OK) {
-            w->cap_wide = 0;
-            return rc;
+        // growing frees first, so there is none until both have grown
+        w->cap_wide = 0;
+        for (uint64_t** p : {&w->sa, &w->sb}) {
+            size_t c = 0;
+            if ((rc = rl_grow(p, &c, (size_t)widest * 5, "subtree sums")) != YX_OK) return rc;
         }
         w->cap_wide = widest;
     }
