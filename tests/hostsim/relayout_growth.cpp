@@ -137,7 +137,10 @@ int main() {
         g_fail_bytes = (size_t)90 * 5 * 8;
         g_fail_nth = nth;
         g_emits = g_bad = 0;
+        uint32_t *const recs0 = recs, *const lod0 = lod;
+        const size_t cap0 = cap;
         expect(layout(w, 200, 90, &recs, &lod, &cap) == YX_ERR_OOM && g_emits == 0, "a wider tree without memory");
+        expect(recs == recs0 && lod == lod0 && cap == cap0, "the records in use after it");
         g_fail_nth = 0;
         expect(layout(w, 200, 50, &recs, &lod, &cap) == YX_OK && g_emits == 3, "the first tree again");
         expect(!g_bad, "its kernels' sums");

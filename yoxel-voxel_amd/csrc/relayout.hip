@@ -461,7 +461,19 @@ int gpu_relayout(const uint32_t* d_vox, uint32_t nn, uint32_t root, void* stream
     w->levels = (int)levels;
     if (depth == 0) return YX_OK;  // no leaf anywhere: nothing to hit
 
-    // the caller's record arrays, grown only when too small
+    // bottom-up subtree sums: two buffers of 5 u64 per node of the widest level
+    if (w->cap_wide < widest) {
+        // growing frees first, so there is none until both have grown
+        w->cap_wide = 0;
+        for (uint64_t** p : {&w->sa, &w->sb}) {
+            size_t c = 0;
+            if ((rc = rl_grow(p, &c, (size_t)widest * 5, "subtree sums")) != YX_OK) return rc;
+        }
+        w->cap_wide = widest;
+    }
+
+    // the caller's record arrays, grown only when too small, and last: after a
+    // failure the caller goes on with the records that it has
     if (*cap_io < total || !*recs_io || !*lod_io) {
         uint32_t *nr = nullptr, *nl = nullptr;
         if (hipMalloc((void**)&nr, total * 8u) != hipSuccess)
@@ -478,16 +490,6 @@ int gpu_relayout(const uint32_t* d_vox, uint32_t nn, uint32_t root, void* stream
     }
     uint2* d_recs = reinterpret_cast<uint2*>(*recs_io);
     uint32_t* d_lod = *lod_io;
-    // bottom-up subtree sums: two buffers of 5 u64 per node of the widest level
-    if (w->cap_wide < widest) {
-        // growing frees first, so there is none until both have grown
-        w->cap_wide = 0;
-        for (uint64_t** p : {&w->sa, &w->sb}) {
-            size_t c = 0;
-            if ((rc = rl_grow(p, &c, (size_t)widest * 5, "subtree sums")) != YX_OK) return rc;
-        }
-        w->cap_wide = widest;
-    }
     uint64_t *sa = w->sa, *sb = w->sb;
     for (int q = (int)levels; q-- > 0;) {
         // a level's nodes are this many levels above the leaves at most
