@@ -536,7 +536,9 @@ int yx_compositor_last_stats(const yx_compositor* c, uint64_t* records, uint64_t
  * of their first appearance in the list, get the lowest free slots in
  * increasing order; bricks that have one keep it. The reference fills the
  * least-used slices of a 3D texture pool; this pool is one linear array.
- * Calls on one pool must not overlap. */
+ * Calls on one pool must not overlap. alloc and release wait on the host for
+ * all of their work; update waits for the check of its list, and its copy,
+ * ordered on `stream`, may still be running when the call returns. */
 typedef struct yx_brick_pool yx_brick_pool;
 /* The table may already map bricks to slots (YX_ERR_FORMAT if a slot is used
  * twice or lies beyond num_slots). */

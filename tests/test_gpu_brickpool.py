@@ -138,6 +138,29 @@ def test_pools_of_many_slots(yx, oracle_mod, cuda, cap):
     assert np.array_equal(params.cpu().numpy(), orc.params)
 
 
+def test_update_returns_before_its_copy(yx, cuda):
+    """update waits for its check alone; the bricks' copy (256 MB here) runs on
+    behind the host. A busy host may find it done by the time it looks, so one
+    of several calls is enough."""
+    torch = cuda
+    dev = torch.device("cuda", 0)
+    grid, brick = 256, 8
+    nb = (grid // brick) ** 3
+    bricks = torch.arange(nb, dtype=torch.int32, device=dev)
+    table = torch.full((nb,), -1, dtype=torch.int32, device=dev)
+    params = torch.zeros((nb * brick ** 3, 4), dtype=torch.float32, device=dev)
+    values = torch.ones_like(params)
+    pool = yx.composite.BrickPool(table, params, grid, brick)
+    pool.alloc(bricks)
+    behind = []
+    for _ in range(10):
+        torch.cuda.synchronize()
+        pool.update(bricks, values)
+        behind.append(not torch.cuda.current_stream().query())
+    assert any(behind)
+    assert torch.equal(params, values)
+
+
 def test_existing_table_and_bad_table(yx, cuda):
     torch = cuda
     vol = yx.composite.Volume(64, 8, occupancy=0.2, seed=3)
