@@ -312,10 +312,11 @@ typedef struct yx_tuning {
                              or 256, 512 (replay kernel)                        */
     int32_t tile_w;       /* ray packet (queue tile) width in pixels, power of 2 */
     int32_t tile_h;       /* ray packet height, power of 2; tile_w*tile_h <= 4096 */
-    int32_t refill_min;   /* idle lanes before a wave takes new rays, 1..64     */
+    int32_t refill_min;   /* waiting lanes before a wave serves them, 1..64     */
     int32_t queues;       /* ray queues, 1..64 (8 = one per XCD)                */
     int32_t window;       /* stack levels kept in registers: 0..6 (stack kernel
-                             uses 0, 2, 4, 6; replay kernel 0, 1, 2)           */
+                             uses 0, 2, 4, 6, and 2 for 0 when a camera or light
+                             is not finite; replay kernel 0, 1, 2)             */
     int32_t waves_per_cu; /* persistent launch size; 0 = occupancy limit        */
     int32_t lds_levels;   /* stack kernel, single scene: node records of tree
                              levels 0..lds_levels-1 staged in LDS per workgroup
@@ -326,8 +327,8 @@ int yx_renderer_get_tuning(const yx_renderer* r, yx_tuning* tuning);
 
 /* ---- autotuner ------------------------------------------------------------
  * Coordinate descent over the tuning space of the stack kernel: ray packet
- * shape (tile_w x tile_h), queue chunk (refill_min: idle lanes a wave gathers
- * before it takes that many ray ids with one atomic), register window (levels
+ * shape (tile_w x tile_h), refill threshold (refill_min: lanes that wait before
+ * a wave gives them new rays and does their once-per-ray work), register window (levels
  * kept in registers; the rest of the traversal stack is LDS-resident),
  * workgroup size and queue count. Each candidate renders `reps` timed frames
  * (after one untimed one) into `out` on `stream`; the best is kept in the
@@ -419,7 +420,10 @@ void yx_batch_destroy(yx_batch* b);
  * yx_renderer_set_scene). Replaces any previous scenes and jobs. */
 int yx_batch_set_scenes(yx_batch* b, const yx_scene* const* scenes, int32_t n);
 /* Sets the jobs; total_pixels (may be NULL) receives the output size. Calling
- * it again with only cameras and lights changed keeps the captured graph. */
+ * it again with only cameras and lights changed keeps the captured graph,
+ * unless the first or last camera or light that is not finite comes or goes:
+ * a batch that holds one is traced by the kernel with a register window of two
+ * levels, which treats NaN as the recursion does and is slower. */
 int yx_batch_set_jobs(yx_batch* b, const yx_batch_job* jobs, int32_t n, uint64_t* total_pixels);
 int yx_batch_job_offset(const yx_batch* b, int32_t job, uint64_t* first_pixel);
 int yx_batch_set_tuning(yx_batch* b, const yx_tuning* tuning); /* stack kernel only */

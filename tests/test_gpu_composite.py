@@ -90,8 +90,8 @@ def test_uneven_bricks_and_dense_volume(yx, oracle_mod, cuda):
 
 @pytest.mark.parametrize("grid,brick,occupancy", [(16, 1, 0.5), (32, 2, 0.6), (64, 16, 0.5)])
 def test_brick_sizes(yx, oracle_mod, cuda, grid, brick, occupancy):
-    # bricks of 1 and 2 voxels go through the per-slot reduction with 1 and 8
-    # voxel sums per slot; 16^3 bricks through the whole-key sort and run sums
+    # 512 bricks of 1 voxel or 64 of 2^3 share a cell of sums; a 16^3 brick is
+    # eight cells
     run_parity(yx, oracle_mod.CompositeOracle(), cuda, grid, brick, occupancy, 5, 2, 24, 20, nsel=64)
 
 
@@ -216,7 +216,7 @@ def test_backward_capacity(yx, cuda, brick):
     """The record total stays on the device. A reserved capacity gives the same
     bits as a backward that sized its own workspace; a capacity below the total
     gives a NaN gradient and a reported error, and the next call grows the
-    workspace and is exact again. brick 8 reduces per slot, 16 by whole keys."""
+    workspace and is exact again. A brick of 8^3 is one cell of sums, of 16^3 eight."""
     torch = cuda
     grid, w, h = 64, 40, 32
     v, views, table, params, vd = setup_case(yx, torch, grid, brick, 0.4, 11, 3, w, h)

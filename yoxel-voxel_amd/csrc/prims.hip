@@ -385,8 +385,11 @@ __global__ __launch_bounds__(kSortThreads) void prim_rs_downsweep(const K* keys_
 // of the current device, and never more than kSortMaxBlocks, which sizes the
 // workspace. Fewer blocks mean fewer scattered histogram entries (the
 // upsweep's 256 stores and the downsweep's 256 loads per block), more mean
-// better balance; on composite_512's 82 M records 16 per CU (about 5 tiles a
-// block) measured best of 4, 6, 8, 12, 16, 24 and 32.
+// better balance. With 82 M keys 16 per CU (about 5 tiles a block) measured
+// best of 4, 6, 8, 12, 16, 24 and 32; with the 16 M segments that the
+// compositor's adjoint sorts (under a capacity of 102 M, which the block count
+// follows: a tile a block) 4 / 8 / 16 / 32 take 3,055 / 3,040 / 3,050 / 3,075
+// us a whole step.
 constexpr uint32_t kSortBlocksPerCU = 16;
 constexpr uint32_t kSortMaxBlocks = 8192;
 uint32_t resident_sort_blocks() {
